@@ -38,6 +38,7 @@
 #include <vector>
 
 #include "../../include/moldy_hip.h"
+#include "mdk_brick.h"
 #include "mdk_internal.h"
 #include "mdk_wave.h"
 
@@ -1227,7 +1228,7 @@ __global__ void __launch_bounds__(64) k_full_list_blk(
 // workgroup of NT threads each and at most one atom a thread.  The pair passes
 // keep the atoms of a brick and of the cells around it (6x6x6) in LDS, so the
 // list holds LDS byte offsets of 16 bits instead of atom indices and cell codes.
-//   binfo[b]   first atom, atoms, staged atoms of brick b
+//   binfo[b]   first atom, atoms, staged atoms of brick b (brick_extent)
 //   bstage     b's staged atoms (brick_cap each): index | cell h << BRICK_H_SHIFT,
 //              h = hx + 6 hy + 36 hz of the 6x6x6 cells; the brick's own atoms
 //              come first, in order
@@ -1238,10 +1239,6 @@ __global__ void __launch_bounds__(64) k_full_list_blk(
 // Entries are found as in k_full_list_blk, a row of three cells at a time, as a
 // bit mask of hits, so that the lanes append in step; the masks of the skin's
 // entries wait in LDS until the others are written.
-#define BRICK_THREADS_MAX 512
-#define BRICK_CELLS 216
-#define BRICK_CAP_MAX 2560  // staged atoms: 40 KB of LDS, below 64 KB with the list kernel's masks
-#define BRICK_H_SHIFT 24
 struct Quad16 {
   unsigned a, b;
   int m;
@@ -1309,13 +1306,13 @@ __global__ void __launch_bounds__(NT) k_brick_list(const float4 *__restrict__ p4
   }
   if (t < BRICK_CELLS) hoff[t] = off;
   if (t == 0) hoff[BRICK_CELLS] = total;
-  const bool fits = total < cap && own <= NT;
+  const int4 info = brick_extent(a0, own, total, NT, cap);
   if (t == 0) {
-    binfo[bi] = fits ? make_int4(a0, own, total, 0) : make_int4(a0, 0, 0, 0);
+    binfo[bi] = info;
     if (own > NT) atomicMax(&flags[1], own);
     if (own > 0 && total >= cap) atomicMax(&flags[3], total + 1);
   }
-  if (!fits || own == 0) return;  // uniform
+  if (info.y == 0) return;  // uniform: no bstage words, and none counted
   // centre of the staged cell from the brick's centre, in FP32 positions (the
   // rounding is immaterial against the skin); .w = LDS offset in the pair passes
   const double fx = (hx - 2.5) * pg.ix, fy = (hy - 2.5) * pg.iy, fz = (hz - 2.5) * pg.iz;
