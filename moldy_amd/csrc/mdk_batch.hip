@@ -83,9 +83,10 @@ int berr(int code, const char *fmt, ...) {
 struct CellMeta {
   int a0, nc, tile0, ntile;
   int nx, ny, nz, rows;
-  int est0;   // first entry of the cell's record offsets in est
-  int rec0;   // first candidate record
-  int pad0, pad1;
+  int est0;     // first entry of the cell's record offsets in est
+  int rec0;     // first candidate record
+  float ext;    // largest sum over cell vectors of a Cartesian component's magnitude
+  int pad;
 };
 
 struct Tile {
@@ -115,7 +116,7 @@ struct BatchArgs {
   double *out_f;         // 3 per caller atom, Cartesian forces
   int *flags;            // [0] max neighbour count seen when over capacity
   int *flags_out;        // host-mapped copy, written by k_cells
-  float rc2f;            // list radius squared, 1e-4 A past the outermost knot (pairs beyond it add exact zeros)
+  double rc;             // interaction range (outermost knot)
   const float *fetab;    // FP32 form: V, V', phi' interval table of the knots
   // adjoint
   const double *e_in;    // per cell: dL/dE_c (vector-Jacobian product) or target E_c (loss)
@@ -285,10 +286,47 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// A walk finds partners by FP32 positions in the whole cell, whose rounding grows
+// with the cell: a separation is off by at most 16 half-ulps of the extent (rows: 2
+// for the record, 1 for the atom, 1 for the shifts, 5 for adding those, times
+// sqrt(3); less by fractions), below 1e-6 of it, and by 1e-5 A of the FP32 square.
+// So lists end that much past the range, at least 1e-4 A (pairs beyond the range add
+// exact zeros).  FP64 lists end at the range: the few partners that are not inside it
+// for certain are tested again, in FP64 and by the separation that the passes form.
+// us per pass with one FP32 test against 1e-4 A : so -- 48 cells in FP64, list and
+// adjoint 298 : 305; 1024 cells in FP32, loss and gradient 472 : 473.
+#define LIST_MARGIN 1e-4
+#define LIST_ROUND 1e-6
+template <typename T> struct Range {
+  float cand2, sure2;  // squares: candidates below, and in range for certain below
+  double rc2;
+  const double4 *pc;
+  double4 pi;
+  const Shifts<T> &S;
+  __device__ __forceinline__ Range(const BatchArgs &A, const TileView &V, const Shifts<T> &S_) : S(S_) {
+    const double off = LIST_ROUND * V.m.ext + 1e-5, c = A.rc + fmax(LIST_MARGIN, off), u = fmax(A.rc - off, 0.0);
+    cand2 = (float)(c * c);
+    if constexpr (sizeof(T) == 8) {
+      sure2 = (float)(u * u);
+      rc2 = A.rc * A.rc;
+      pc = A.pos4 + V.m.a0;
+      pi = pc[V.active ? V.il : 0];
+    }
+  }
+  // whether candidate j with the FP32 square r2 belongs to the list
+  __device__ __forceinline__ bool holds(float r2, int j, int code) const {
+    if constexpr (sizeof(T) == 8) {
+      if (r2 < sure2) return true;
+      double x, y, z;
+      pair_sep(pi, pc[j], S, code, x, y, z);
+      return x * x + y * y + z * z < rc2;
+    }
+    return true;
+  }
+};
+
 // Appends the partners of this lane's atom to its list (a whole wave calls; lanes
-// past the tile's atoms only help to stage).  The test takes FP32 positions and
-// the list radius ends 1e-4 A past the outermost knot: its rounding (below 1e-5 A)
-// can only add or drop pairs whose terms are exactly zero.
+// past the tile's atoms only help to stage).
 // The candidate records of a plane of rows pass through LDS in windows of at most
 // LIST_WIN (a plane's rows of the tile's sub-cells mostly fit one), read in order,
 // and each lane tests those of its three rows.  Read by every lane for itself, 16
@@ -306,7 +344,9 @@ __device__ __forceinline__ int wave_max_i(int v) {
   for (int o = 1; o < 64; o <<= 1) v = max(v, __shfl_xor(v, o, 64));
   return __builtin_amdgcn_readfirstlane(v);
 }
-__device__ __forceinline__ void walk_rows(const BatchArgs &A, const TileView &V, float4 *win, ListOut &out) {
+template <typename T>
+__device__ __forceinline__ void walk_rows(const BatchArgs &A, const TileView &V, const Range<T> &N, float4 *win,
+                                          ListOut &out) {
   const double *b = A.box + 9 * (size_t)V.t.cell;
   const int lane = threadIdx.x & 63;
   const size_t a = (size_t)V.m.a0 + (V.active ? V.il : 0);
@@ -359,10 +399,11 @@ __device__ __forceinline__ void walk_rows(const BatchArgs &A, const TileView &V,
           const int m = min(32, end - c0);
           const float4 *q = win + (c0 - w0);
           unsigned hit = 0;
-          auto test = [&](const float4 &p, int k) {
+          auto sep2 = [&](const float4 &p) {
             const float ex = qx - p.x, ey = qy - p.y, ez = qz - p.z;
-            hit |= ex * ex + ey * ey + ez * ez < A.rc2f ? 1u << k : 0u;
+            return ex * ex + ey * ey + ez * ez;
           };
+          auto test = [&](const float4 &p, int k) { hit |= sep2(p) < N.cand2 ? 1u << k : 0u; };
           int k = 0;
           for (; k + 4 <= m; k += 4) {  // four LDS reads in flight
             const float4 q0 = q[k], q1 = q[k + 1], q2 = q[k + 2], q3 = q[k + 3];
@@ -373,10 +414,12 @@ __device__ __forceinline__ void walk_rows(const BatchArgs &A, const TileView &V,
           }
           for (; k < m; k++) test(q[k], k);
           while (hit) {
-            const int h = __builtin_ctz(hit), c = c0 + h, j = __float_as_int(q[h].w);
+            const int h = __builtin_ctz(hit), c = c0 + h;
+            const float4 p = q[h];
+            const int j = __float_as_int(p.w);
             hit &= hit - 1;
             const int code = base + (c >= m1[y] ? 1 : 0) + (c >= m2[y] ? 1 : 0);
-            if (j != V.il) out.put(j | (code << NB_CODE_SHIFT));
+            if (j != V.il && N.holds(sep2(p), j, code)) out.put(j | (code << NB_CODE_SHIFT));
           }
         }
       }
@@ -386,7 +429,8 @@ __device__ __forceinline__ void walk_rows(const BatchArgs &A, const TileView &V,
 // Any grid (some dimension with one sub-cell): the nearest image of the
 // fractional separation.  An in-range pair's nearest image is the one its
 // sub-cell offset names, since the cell is wider than twice the range.
-__device__ __forceinline__ void walk_any(const BatchArgs &A, const TileView &V, ListOut &out) {
+template <typename T>
+__device__ __forceinline__ void walk_any(const BatchArgs &A, const TileView &V, const Range<T> &N, ListOut &out) {
   const double *b = A.box + 9 * (size_t)V.t.cell;
   const size_t a = (size_t)V.m.a0 + V.il;
   const int nx = V.m.nx, ny = V.m.ny, nz = V.m.nz;
@@ -418,9 +462,10 @@ __device__ __forceinline__ void walk_any(const BatchArgs &A, const TileView &V, 
             const float x = bf[0] * ex + bf[3] * ey + bf[6] * ez, y = bf[1] * ex + bf[4] * ey + bf[7] * ez,
                         z = bf[2] * ex + bf[5] * ey + bf[8] * ez;
             const int j = __float_as_int(q[u].w);
-            if (x * x + y * y + z * z < A.rc2f && c + u < hi && j != V.il) {
+            const float r2 = x * x + y * y + z * z;
+            if (r2 < N.cand2 && c + u < hi && j != V.il) {
               const int code = (rx ? ox : (int)tx) + 3 * (ry ? oy : (int)ty) + 9 * (rz ? oz : (int)tz) + 13;
-              out.put(j | (code << NB_CODE_SHIFT));
+              if (N.holds(r2, j, code)) out.put(j | (code << NB_CODE_SHIFT));
             }
           }
         }
@@ -448,8 +493,9 @@ __global__ void __launch_bounds__(BLOCK) k_list(BatchArgs A, PotDev P) {
   const int lane = threadIdx.x & 63;
   int4 *nb = A.nbr + (size_t)max(V.index, 0) * (A.maxnb / 4) * TILE + lane;
   ListOut out = {nb, A.maxnb, 0, 0, 0, 0, 0};
-  if (V.m.rows) walk_rows(A, V, win[threadIdx.x >> 6], out);
-  else if (V.active) walk_any(A, V, out);
+  const Range<T> N(A, V, S);
+  if (V.m.rows) walk_rows<T>(A, V, N, win[threadIdx.x >> 6], out);
+  else if (V.active) walk_any<T>(A, V, N, out);
   if (V.active) {
     const size_t a = (size_t)V.m.a0 + V.il;
     int cnt = out.cnt;
@@ -902,7 +948,7 @@ BatchArgs args_of(mdk_batch *b) {
   A.s = b->s; A.perm = b->perm; A.rec = b->rec; A.pos4 = b->pos4; A.p4f = b->p4f; A.daf = b->daf; A.nbr = b->nbr;
   A.numn = b->numn; A.rho = b->rho; A.part = b->part; A.out_e = b->out_e; A.out_w = b->out_w; A.out_f = b->out_f;
   A.flags = b->flags; A.flags_out = b->flags_map;
-  A.rc2f = (float)((b->rc + 1e-4) * (b->rc + 1e-4));
+  A.rc = b->rc;
   A.fetab = b->fetab;
   A.e_in = b->e_tgt; A.f_in = b->f_tgt; A.gvec = b->gvec; A.ecell = b->ecell; A.part_g = b->part_g;
   A.out_loss = b->out_loss; A.f_weight = 0.1 / (double)b->natom;
@@ -1049,8 +1095,11 @@ int plan(mdk_batch *b, double rgrid) {
     }
     const int a0 = b->h_off[c], nc = b->h_off[c + 1] - a0, nsc = g[0] * g[1] * g[2];
     CellMeta &m = meta[c];
+    double ext = 0.0;
+    for (const double *B = &b->h_box[9 * (size_t)c], *r = B; r < B + 3; r++)
+      ext = std::max(ext, fabs(r[0]) + fabs(r[3]) + fabs(r[6]));
     m = CellMeta{a0, nc, (int)tiles.size(), (nc + TILE - 1) / TILE, g[0], g[1], g[2],
-                 g[0] >= 3 && g[1] >= 3 && g[2] >= 3 ? 1 : 0, (int)est.size(), (int)rsrc.size(), 0, 0};
+                 g[0] >= 3 && g[1] >= 3 && g[2] >= 3 ? 1 : 0, (int)est.size(), (int)rsrc.size(), (float)ext, 0};
     for (int i = 0; i < nc; i += TILE) tiles.push_back(Tile{c, a0 + i, std::min(TILE, nc - i), i});
     key.resize(nc);
     start.assign(nsc + 1, 0);
