@@ -198,7 +198,11 @@ int mdk_velocityverlet(void *h);
 int mdk_update_therm_avs(void *h, double *s1, double *s2, double *s3);
 /* nsteps MD steps of the moldin loop (velocityverlet, update_therm_avs,
  * KE/TE/H/TH, relink when ntc==0) without host round trips; if trace is not
- * NULL it receives per step {pe, ke, te, h, th, vol} (6*nsteps doubles). */
+ * NULL it receives per step {pe, ke, te, h, th, vol} (6*nsteps doubles).
+ * A call that an error stops between two steps (MDK_ERR_SKIN) leaves the forces,
+ * densities and energies of its last step, and the positions drifted to the next
+ * one; in a box that does not move (ivol 1, 2, 3, 5) TK, TP, FB, S1 and S2 are
+ * formed by a call's last step only and are then those of the call before. */
 int mdk_md_steps(void *h, int nsteps, double *trace);
 /* Number of full-list rebuilds performed so far and the current full-list
  * pair count (sum over atoms, each pair counted twice). */

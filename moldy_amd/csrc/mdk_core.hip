@@ -4064,6 +4064,21 @@ static int flush_ride(mdk_ctx *c) {
   return check_launch("k_finish_step");
 }
 
+// FX..FZ of the last step of a call that stopped after one with a fused kick, which
+// forms no forces for memory: from the packed records that its force pass read (the
+// alternate ones by now, F' included) over the same list.
+static int last_forces(mdk_ctx *c) {
+  const bool fp64 = !lean_path(c), kin = c->kin_fresh;
+  std::swap(c->p4f, c->p4f_alt);
+  if (fp64) std::swap(c->pos4, c->pos4_alt);
+  c->kin_fresh = true;  // no sums are wanted
+  const int rc = launch_force(c);
+  c->kin_fresh = kin;
+  std::swap(c->p4f, c->p4f_alt);
+  if (fp64) std::swap(c->pos4, c->pos4_alt);
+  return rc;
+}
+
 // Waits until the device has written the stamp: a spin on host-mapped memory
 // (an event wait wakes the host microseconds later); a stream that failed or
 // drained without writing it ends the wait.
@@ -5300,8 +5315,19 @@ extern "C" int mdk_md_steps(void *h, int nsteps, double *trace) {
     // relink when the reference's ntc counter wraps (moldin.F90:791)
     if (rc == MDK_OK && c->ntc == 0 && !c->drifted) rc = relink_in_loop(c);
   }
+  // the list is still the one of a fused last step if that step's sums are pending
+  // and no rebuild has begun
+  const bool fused = c->ride.kind == 2 && c->list_valid && !c->list_pending;
   const int rf = flush_ride(c);  // the last step's sums (also after a failed step)
-  if (rc != MDK_OK) return rc;
+  if (rc != MDK_OK) {
+    if (fused) {
+      char msg[sizeof(g_err)];
+      memcpy(msg, g_err, sizeof(msg));
+      if (last_forces(c) == MDK_OK) hipStreamSynchronize(c->stream);
+      set_err(rc, "%s", msg);
+    }
+    return rc;
+  }
   RCK(rf);
   if (trace && nsteps > 0)
     HIPCK(hipMemcpyAsync(trace, c->trace_dev, sizeof(double) * 6 * (size_t)nsteps, hipMemcpyDeviceToHost, c->stream));
