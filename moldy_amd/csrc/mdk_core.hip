@@ -4185,11 +4185,16 @@ static int launch_kick(mdk_ctx *c, int mode, double *trace_row_dev, double *mon,
 
 // force()'s finishing and the half kick of a small system in one launch (the
 // MD loop); the kick's sums stay pending as with a deferred launch_kick.
-// us per NPT step, two kernels : one -- 2000 atoms (FP64) 27.1 : 22.5, 16,000
-// 27.2 : 26.0 (FP32 27.3 : 25.2), 31,250 33.8 : 34.6 (32.5 : 31.9), 39,366
-// 35.9 : 38.3 (32.4 : 35.1): every workgroup folds the partials, which pays
-// while there are few of both.
-#define FIN_KICK_BLOCKS 640
+// Every workgroup folds the partials of every workgroup of the pair passes, so what
+// it saves (a launch and the gap) is lost where the product of the two numbers is
+// large.  us per NPT step, two kernels : one, FP64 (FP32) --
+//   eight lanes per atom  2000 22.2 : 19.3 (22.7 : 20.0)    8192 24.0 : 21.5 (24.5 : 22.4)
+//   four                  16,000 24.3 : 23.1 (24.7 : 23.1)  31,250, product 60,000: 28.8 : 28.3 (27.3 : 27.3)
+//                         39,366, 95,000: 31.0 : 31.2 (28.6 : 28.7)  47,096, 136,000: 32.0 : 32.6 (29.5 : 30.0)
+//   two                   54,000, 89,000: 32.4 : 32.7 (30.4 : 30.8)  78,608, 189,000: 38.5 : 39.7 (33.9 : 35.2)
+//   one                   128,000, 250,000: 44.0 : 45.9 (39.0 : 40.3)  159,014, 387,000: 53.7 : 54.5 (42.6 : 44.4)
+//   eight, iron_carbon    16,000, 31,500: 32.9 : 32.6  21,296, 56,000: 38.0 : 37.9  27,648, 93,000: 43.0 : 43.9
+#define FIN_KICK_FOLDS 64000
 static int launch_finish_kick(mdk_ctx *c, double *trace_row_dev, double *mon, bool fuse_drift, bool link) {
   const FinForce F = fin_force(c, FIN_VV_THERM);
   BoxState *fin = c->box + next_box(c), *nxt = c->box + next_box(c, 2);
@@ -4392,7 +4397,7 @@ static int md_step(mdk_ctx *c, double *trace_row_dev, int more) {
     c->kin_nb = c->nbp;
   } else {
     RCK(force_body(c, skin_due));
-    if (c->nbp <= FIN_KICK_BLOCKS) {
+    if ((long)c->nblk * c->nbp <= FIN_KICK_FOLDS) {
       RCK(launch_finish_kick(c, trace_row_dev, mon, fuse, link));
     } else {
       RCK(launch_finish(c, FIN_VV_THERM));
