@@ -187,7 +187,8 @@ struct mdk_ctx {
   int *lblocks, nlblocks, lblocks_cap, lblock_g[3], lblock_side;
   // brick list (k_brick_list): its entries and their quads per atom, staged atoms
   // and extents of every brick
-  bool brick, brick_bad;   // the list is one; this handle's bricks do not fit
+  bool brick, brick_bad;   // the list is one; bricks did not fit lately
+  int brick_fit;           // lists planned since a build last changed that or the sizes below (0: none did)
   bool brick_built;        // nbr16, bcnt, bstage and binfo hold a built list
   bool wide_valid;         // nbr, numn hold the brick list's pairs as well (ensure_wide_list)
   uint2 *nbr16;
@@ -3580,8 +3581,16 @@ static int brick_threads(double m) {
 // Whether grid g is listed by bricks; g then has whole bricks where their atoms
 // still fit (524,288 atoms of bcc Fe: 11^3 bricks of 394 atoms instead of 12^3, of
 // which 397 have a cell or two).  The threads are those of the mean brick and a
-// few atoms more, or of the largest brick so far.
+// few atoms more, or of the largest brick lately: what a build that did not fit has
+// taught (fit_bricks) holds for BRICK_RETRY lists, so that a system which was uneven
+// for a while returns to the better form; one that stays uneven builds a list in 32
+// twice.
+#define BRICK_RETRY 32
 static bool plan_bricks(mdk_ctx *c, int g[3]) {
+  if (c->brick_fit && ++c->brick_fit > BRICK_RETRY) {
+    c->brick_fit = c->brick_nt = c->brick_cap = 0;
+    c->brick_bad = false;
+  }
   if (!brick_size(c) || !lean_pot(c) || c->lanes != 1 || c->brick_bad) return false;
   const int f[3] = {g[0] & ~3, g[1] & ~3, g[2] & ~3};
   auto atoms = [&](const int *q) { return 64.0 * c->n / ((double)q[0] * q[1] * q[2]); };
@@ -3624,6 +3633,7 @@ static int ensure_brick(mdk_ctx *c, double per_cell) {
 static void fit_bricks(mdk_ctx *c, const volatile int *fl) {
   const int nt = brick_threads(fl[1]);
   if (nt == 0 || fl[3] > BRICK_CAP_MAX) c->brick_bad = true;
+  c->brick_fit = 1;
   c->brick_nt = std::max(c->brick_nt, nt);
   if (fl[3]) c->brick_cap = std::min(BRICK_CAP_MAX, fl[3] + fl[3] / 16);
 }
