@@ -211,7 +211,8 @@ int mdk_stats(void *h, long *rebuilds, long *full_pairs);
 /* Timing: per-kernel-class HIP-event accumulators on the handle's stream for
  * classes {0 drift, 1 density, 2 force, 3 kick, 4 rebuild}.  mask selects the
  * classes to record (bit k = class k; MDK_TIMING_ALL every class, 0 stops);
- * each recorded launch adds two events to the stream.  mdk_timing_read
+ * each recorded launch adds two events to the stream.  In a box that does not move
+ * the kick of the steps inside a call is part of the force launch.  mdk_timing_read
  * returns total milliseconds and launch counts per class. */
 #define MDK_TIMING_ALL 0x1F
 int mdk_timing(void *h, int mask);
@@ -234,6 +235,10 @@ int mdk_batch_create(void **handle, int ncell, const int *natoms, const double *
                      const double *s, int precision);
 int mdk_batch_destroy(void *handle);
 const char *mdk_batch_last_error(void);
+/* The first potential, and one whose range grows by more than 2 % or falls below 0.8
+ * of the planned sub-cells, lays the cells out again: it allocates device memory and
+ * waits for launches in flight.  The layout decides the order of sums over atoms, so
+ * results with one potential agree bit for bit while it stays. */
 int mdk_batch_set_potential(void *h, int nv, const double *av, const double *rv, int np,
                             const double *ap, const double *rp);
 /* workgroup size of the passes over atoms (64, 128, 256 or 512), workgroups per
@@ -244,7 +249,8 @@ int mdk_batch_synchronize(void *h);
 /* energy[ncell] eV; virial[6*ncell] = sum over pairs r r^T fp (xx yy zz xy xz yz),
  * stress = -virial/volume; forces[3*natom] Cartesian eV/A; rho[natom]; any may be NULL */
 int mdk_batch_results(void *h, double *energy, double *virial, double *forces, double *rho);
-/* autotuner over the block size (best of reps replays) */
+/* autotuner over the block size (best of reps replays); best_wgpc receives the
+ * setting as it is */
 int mdk_batch_tune(void *h, int reps, int *best_block, int *best_wgpc, double *best_ms);
 int mdk_batch_time(void *h, int reps, double *ms_avg);
 int mdk_batch_info(void *h, int *natom, int *block, int *wg_per_cu, long *pairs);
@@ -275,7 +281,8 @@ int mdk_batch_time_loss_grad(void *h, int reps, double *ms_avg);
  * loss (1 double) and grad (2 nv + 2 np doubles) are DEVICE pointers, written
  * asynchronously on the batch's stream; mdk_batch_synchronize before reading
  * them (it also reports a neighbour-capacity overflow).  A batch with more than
- * MDK_NOALLOC_MAX_CELLS cells gives MDK_ERR_BAD_ARG.  Results equal
+ * MDK_NOALLOC_MAX_CELLS cells gives MDK_ERR_BAD_ARG (a limit of the interface, kept
+ * for callers that size by it; the workspace is the handle's own).  Results equal
  * mdk_batch_loss_grad's bit for bit; the batch's graph is not used. */
 #define MDK_NOALLOC_MAX_CELLS 8192
 int mdk_batch_loss_grad_noalloc(void *h, double *loss, double *grad);

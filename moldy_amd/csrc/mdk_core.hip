@@ -227,9 +227,7 @@ struct mdk_ctx {
   int nblk;
   int lanes, nbp;          // lanes per atom of the pair passes (pair_lanes) and their blocks
   int part_cap;            // blocks the partial arrays hold
-  // host-mapped monitor ring, MON_STRIDE doubles per step slot (4 slots):
-  // [0] maxdisp2, [1] maxstep2, [2..10] B0 after the step, [11] full-list
-  // overflow flag, [12] grid-too-coarse flag
+  // host-mapped monitor ring: four step slots of MON_STRIDE doubles (layout there)
   double *mon_host, *mon_dev;
   double b0_lag[9];        // B0 of a completed step (from the monitor ring)
   long b0_lag_step;        // its step index, -1 when none
@@ -4255,8 +4253,8 @@ static int launch_drift(mdk_ctx *c) {
 
 // Reads the monitor sample of step s-3 (its kernels have completed or the
 // host waits for them): the box for the next grid plan and the skin bound.
-// In the MD loop a step's sample is finished by the next step's force
-// finishing kernel, so the host stays about two steps ahead of the GPU.
+// In the MD loop a step's sample is completed by the next step's density pass,
+// so the host stays about two steps ahead of the GPU.
 static int poll_monitor(mdk_ctx *c, const double **sample) {
   const long s = c->step_counter;
   *sample = nullptr;

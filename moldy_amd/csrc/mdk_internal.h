@@ -8,9 +8,14 @@
 // 3x3 tensors are Fortran column-major: T(i,j) == t[(j-1)*3 + (i-1)].
 #define TT(a, i, j) (a)[((j)-1) * 3 + ((i)-1)]
 
-// Box and thermodynamic state of one system, resident on the device.  Two
-// copies exist; a step reads copy `cur` in its drift kernel and writes the
-// advanced box into the other copy, which every later kernel of the step uses.
+// Box and thermodynamic state of one system, resident on the device, in four
+// copies used in turn (mdk_ctx::cur).  A kernel in which every workgroup reads the
+// current copy writes its results into later ones: a drift, a predictor and a kick
+// with the next drift the advanced box into cur + 1; a kick that also finishes the
+// forces the finished box into cur + 1 and the advanced one into cur + 2, which no
+// workgroup of that launch reads.  The step's own sums follow in the next density
+// pass, into the finished copy and the advanced one: before any later kernel writes
+// either again.  Steps in a fixed box between two others of a call stay on one copy.
 struct BoxState {
   double b0[9], b1[9], b2[9], b3[9];  // b3: box jolt of the predictor-corrector
   double tk[9], tc[9], tg[9], tp[9], tginv[9], tgdot[9], tgid[9], fb[9];
