@@ -188,7 +188,7 @@ struct mdk_ctx {
   // brick list (k_brick_list): its entries and their quads per atom, staged atoms
   // and extents of every brick
   bool brick, brick_bad;   // the list is one; bricks did not fit lately
-  int brick_fit;           // lists planned since a build last changed that or the sizes below (0: none did)
+  int brick_wait;          // lists planned since then
   bool brick_built;        // nbr16, bcnt, bstage and binfo hold a built list
   bool wide_valid;         // nbr, numn hold the brick list's pairs as well (ensure_wide_list)
   uint2 *nbr16;
@@ -3579,16 +3579,14 @@ static int brick_threads(double m) {
 // Whether grid g is listed by bricks; g then has whole bricks where their atoms
 // still fit (524,288 atoms of bcc Fe: 11^3 bricks of 394 atoms instead of 12^3, of
 // which 397 have a cell or two).  The threads are those of the mean brick and a
-// few atoms more, or of the largest brick lately: what a build that did not fit has
-// taught (fit_bricks) holds for BRICK_RETRY lists, so that a system which was uneven
-// for a while returns to the better form; one that stays uneven builds a list in 32
-// twice.
+// few atoms more, or of the largest brick so far (a liquid's, which needs its size
+// again and again: forgotten every 32 lists it cost 1.4 % of 3,456,000 atoms' steps).
+// Bricks that did not fit any workgroup are tried again after BRICK_RETRY lists, so
+// that a system which was uneven for a while returns to the better form; one that
+// stays so builds a list in 32 twice.
 #define BRICK_RETRY 32
 static bool plan_bricks(mdk_ctx *c, int g[3]) {
-  if (c->brick_fit && ++c->brick_fit > BRICK_RETRY) {
-    c->brick_fit = c->brick_nt = c->brick_cap = 0;
-    c->brick_bad = false;
-  }
+  if (c->brick_bad && ++c->brick_wait > BRICK_RETRY) c->brick_bad = false;
   if (!brick_size(c) || !lean_pot(c) || c->lanes != 1 || c->brick_bad) return false;
   const int f[3] = {g[0] & ~3, g[1] & ~3, g[2] & ~3};
   auto atoms = [&](const int *q) { return 64.0 * c->n / ((double)q[0] * q[1] * q[2]); };
@@ -3630,8 +3628,10 @@ static int ensure_brick(mdk_ctx *c, double per_cell) {
 // after a build in which a brick's atoms (fl[1]) or their surroundings (fl[3]) did not fit
 static void fit_bricks(mdk_ctx *c, const volatile int *fl) {
   const int nt = brick_threads(fl[1]);
-  if (nt == 0 || fl[3] > BRICK_CAP_MAX) c->brick_bad = true;
-  c->brick_fit = 1;
+  if (nt == 0 || fl[3] > BRICK_CAP_MAX) {
+    c->brick_bad = true;
+    c->brick_wait = 0;
+  }
   c->brick_nt = std::max(c->brick_nt, nt);
   if (fl[3]) c->brick_cap = std::min(BRICK_CAP_MAX, fl[3] + fl[3] / 16);
 }
